@@ -105,7 +105,7 @@ static Carve carve_sizes(int T, int H, int I, int E, int K, int Is) {
   c.pos = r256(P * 4);
   c.hits = r256((size_t)(E + 1) * 4);
   c.sort_ws = moe_sort_ws_bytes((int)P, E);
-  c.tiles = r256((size_t)(1 + 2 * moe_max_mtiles((int)P, E, MOE_GEMM6_BM)) * 4);
+  c.tiles = r256((size_t)(1 + 2 * moe_max_mtiles((int)P, E, MOE_GEMM8_BM)) * 4);
   // f32 rows (GEMV path) or f16 rows plus MOE_GEMM3_BM padding rows (the 160-row down kernels
   // read whole tiles past the last row)
   c.S = r256(std::max(P * I * 4, (P + MOE_GEMM3_BM) * I * 2));
@@ -216,18 +216,32 @@ static bool mfma_gu4_mixed(int path, int H, int I, int gu_fmt, int dn_fmt) {
          !mfma_v2(path, H, I, gu_fmt, dn_fmt);
 }
 
-// Q4_K experts with few rows each (up to kSmallRowsMaxT tokens): the 32-row kernels (gemm6.hip),
-// which keep three K steps of activations and nibbles in flight per item
+// Q4_K experts with few rows each (up to kSmallRowsMaxT tokens) at widths gemm8 does not take: the
+// 32-row kernels (gemm6.hip), which keep three K steps of activations and nibbles in flight per item
 constexpr int kSmallRowsMaxT = 256;
 static bool mfma_small(int path, int T, int H, int I, int gu_fmt, int dn_fmt) {
   return mfma_v2(path, H, I, gu_fmt, dn_fmt) && gu_fmt == MOE_FMT_Q4_K && dn_fmt == MOE_FMT_Q4_K &&
          T <= kSmallRowsMaxT && H >= 512 && I >= 512;
 }
 
+// Few rows per expert at the model's width (gemm8.hip): rows per tile of its gate_up and down, 0 where
+// it does not apply. 16-row tiles up to 256 tokens (8 rows per expert on average), 32-row tiles above
+// (gate_up + Q4_K down at 512 tokens, uniform routing: 126 us, 133 on 16-row tiles), up to where the
+// 160-row kernels' rounded weights, decoded once per tile, catch up: 1024 tokens 179 us against
+// 193 on gemm4, 1536 tokens 243 against 203.
+constexpr int kRegRowsOneT = 256, kRegRowsMaxT = 1024;
+static int mfma_reg_rows(int path, int T, int H, int I, int gu_fmt, int dn_fmt) {
+  if (path != MOE_PATH_MFMA || T > kRegRowsMaxT || !moe_gemm8_gateup_supports(gu_fmt, H, I) ||
+      !moe_gemm8_down_supports(dn_fmt, H, I))
+    return 0;
+  return T <= kRegRowsOneT ? 16 : 32;
+}
+
 // rows per MFMA tile of the first grouped GEMM experts_impl runs (0: a GEMV path)
 static int mfma_tile_rows(int path, int T, int H, int I, int gu_fmt, int dn_fmt) {
   path = pick_path(path, T, gu_fmt, dn_fmt);
   if (path == MOE_PATH_GEMV) return 0;
+  if (const int rr = mfma_reg_rows(path, T, H, I, gu_fmt, dn_fmt)) return rr;
   if (mfma_small(path, T, H, I, gu_fmt, dn_fmt)) return MOE_GEMM6_BM;
   return (mfma_v2(path, H, I, gu_fmt, dn_fmt) || mfma_gu4_mixed(path, H, I, gu_fmt, dn_fmt)) ? MOE_GEMM3_BM
                                                                                            : MOE_GEMM_BM;
@@ -241,7 +255,7 @@ static bool y16_rows(int path, int T, int H, int I, int K, int gu_fmt, int dn_fm
 }
 
 // ints of a tile-list buffer that holds the list of any tile height (the shortest tiles: most)
-static size_t tile_list_ints(int P, int E) { return 1 + 2 * (size_t)moe_max_mtiles(P, E, MOE_GEMM6_BM); }
+static size_t tile_list_ints(int P, int E) { return 1 + 2 * (size_t)moe_max_mtiles(P, E, MOE_GEMM8_BM); }
 
 // tiles_pre: the tile list of mfma_tile_rows(...) rows, already built in a buffer of
 // tile_list_ints(P, E) ints (NULL: built here)
@@ -270,7 +284,8 @@ static int experts_impl(const void* x, int x_dtype, const uint16_t* x16, const v
   const bool v2 = mfma_v2(path, H, I, gu_fmt, dn_fmt);
   const bool gu4 = mfma_gu4_mixed(path, H, I, gu_fmt, dn_fmt);
   const bool small = mfma_small(path, T, H, I, gu_fmt, dn_fmt);
-  const int bm = small ? MOE_GEMM6_BM : (v2 || gu4) ? MOE_GEMM3_BM : MOE_GEMM_BM;
+  const int rr = mfma_reg_rows(path, T, H, I, gu_fmt, dn_fmt);
+  const int bm = rr ? rr : small ? MOE_GEMM6_BM : (v2 || gu4) ? MOE_GEMM3_BM : MOE_GEMM_BM;
   const int max_tiles = moe_max_mtiles(P, E, bm);
   int32_t* tiles = tiles_pre;
   if (!tiles) {
@@ -300,6 +315,10 @@ static int experts_impl(const void* x, int x_dtype, const uint16_t* x16, const v
       if (!c) return moe_set_error(MOE_E_WORKSPACE, "moe_experts: workspace too small");
       MOE_TRY(moe_launch_to_f16(x, x_dtype, (size_t)T * H, c, st));
       x16 = c;
+    }
+    if (rr) {
+      MOE_TRY(moe_launch_gemm8_gateup(x16, gate, up, estride, tiles, max_tiles, bm, offsets, sorted_pairs, K, H, I, S, st));
+      return moe_launch_gemm8_down(S, dn, dn_fmt, (size_t)H * dn_row, tiles, max_tiles, bm, offsets, H, I, y, y16, st, shd);
     }
     if (small) {
       MOE_TRY(moe_launch_gemm6_gateup(x16, gate, up, estride, tiles, max_tiles, offsets, sorted_pairs,
@@ -627,8 +646,8 @@ static int block_forward_impl(const void* x, int x_dtype, int T, int H, int I, i
   // blocks, and the shared down blocks run inside the routed down launch: both grids leave CUs
   // idle at this size, and the fork and join cost more than the shared expert's time left after
   // that overlap.
-  const bool fuse = rpath == MOE_PATH_MFMA && Wt.shared_fmt == MOE_FMT_BF16 && H % 2048 == 0 &&
-                    I_s % 256 == 0 && mfma_small(rpath, T, H, I, gate_up_fmt, down_fmt) &&
+  const bool fuse = rpath == MOE_PATH_MFMA && Wt.shared_fmt == MOE_FMT_BF16 && H % 2048 == 0 && I_s % 256 == 0 &&
+                    (mfma_reg_rows(rpath, T, H, I, gate_up_fmt, down_fmt) || mfma_small(rpath, T, H, I, gate_up_fmt, down_fmt)) &&
                     shared_skinny(path, Wt.shared_fmt, T, H, I_s) && moe_router_chain_supported(T, H, E, K);
   uint16_t* x16 = nullptr;
   bool x16_late = false;
@@ -657,7 +676,7 @@ static int block_forward_impl(const void* x, int x_dtype, int T, int H, int I, i
     d.w0 = reinterpret_cast<const uint16_t*>(ws_down); d.S = ssh; d.y = sraw; d.T = T; d.H = H; d.Is = I_s;
     // the sort and the tile list inside the router launch, by its last group to finish routing
     MoeSortJob sj;
-    if (tiles && bm >= 32 && bm <= 160) {
+    if (tiles && bm >= MOE_GEMM8_BM && bm <= 160) {
       sj.P = P; sj.offsets = offsets; sj.sorted = sorted; sj.pos = pos; sj.hits = hits;
       sj.tiles = tiles; sj.bm = bm;
     }

@@ -69,6 +69,7 @@ int moe_launch_sort(const int32_t* ids, int P, int E, int32_t* offsets, int32_t*
 #define MOE_GEMM_BM 64
 #define MOE_GEMM3_BM 160
 #define MOE_GEMM6_BM 32
+#define MOE_GEMM8_BM 16   // the shortest tiles of any kernel (gemm8.hip: 16 or 32)
 int moe_max_mtiles(int P, int E, int bm = MOE_GEMM_BM);
 int moe_launch_build_tiles(const int32_t* offsets, const int32_t* hit_list, int E, int P,
                            int32_t* tiles, hipStream_t st, int bm = MOE_GEMM_BM);
@@ -151,6 +152,17 @@ int moe_launch_gemm6_gateup(const uint16_t* x16, const void* w_gate, const void*
                             int I, uint16_t* S, hipStream_t st);
 int moe_launch_gemm6_down(const uint16_t* S, const void* w_down, size_t expert_stride,
                           const int32_t* tiles, int max_tiles, const int32_t* offsets, int H, int I,
+                          void* y, int y16, hipStream_t st, const MoeShJob* sh = nullptr);
+// gemm8.hip: the routed GEMMs for few rows per expert, the weights streamed into registers and
+// multiplied as whole numbers: Q4_K gate_up on tiles of bm = 16 or 32 rows (H == 2048), Q4_K / Q5_K
+// down on tiles of any height (in pieces of 16 or 32 rows). sh as moe_launch_gemm6_down's.
+bool moe_gemm8_gateup_supports(int fmt, int H, int I);
+bool moe_gemm8_down_supports(int fmt, int H, int I);
+int moe_launch_gemm8_gateup(const uint16_t* x16, const void* w_gate, const void* w_up, size_t expert_stride,
+                            const int32_t* tiles, int max_tiles, int bm, const int32_t* offsets,
+                            const int32_t* sorted_pairs, int K, int H, int I, uint16_t* S, hipStream_t st);
+int moe_launch_gemm8_down(const uint16_t* S, const void* w_down, int fmt, size_t expert_stride,
+                          const int32_t* tiles, int max_tiles, int bm, const int32_t* offsets, int H, int I,
                           void* y, int y16, hipStream_t st, const MoeShJob* sh = nullptr);
 // shared-expert blocks of the router (gate/up) and down launches for T tokens (32-row token tiles x
 // 16-column / 32-column slabs)

@@ -1045,8 +1045,8 @@ int moe_launch_router_chain(const void* x, int x_dtype, const void* w, int w_dty
   }
   const MoeSortJob sj = srt ? *srt : MoeSortJob{};
   if (sj.P) {
-    if (sj.P != T * 8 || !sj.offsets || !sj.sorted || !sj.pos || !sj.hits || !sj.tiles || sj.bm < 32 || sj.bm > 160)
-      return moe_set_error(MOE_E_ARG, "router_chain: the fused sort needs P = 8 T, 32 <= bm <= 160 and every output");
+    if (sj.P != T * 8 || !sj.offsets || !sj.sorted || !sj.pos || !sj.hits || !sj.tiles || sj.bm < MOE_GEMM8_BM || sj.bm > 160)
+      return moe_set_error(MOE_E_ARG, "router_chain: the fused sort needs P = 8 T, 16 <= bm <= 160 and every output");
   }
   dim3 grid(((T + 15) / 16) * (E / 16) * kChainKS);
   grid.x += (unsigned)job.n;

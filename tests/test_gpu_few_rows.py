@@ -1,0 +1,89 @@
+"""Routed experts with few rows each (16- and 32-row tiles, weights multiplied as whole numbers)
+against the oracle, at the edges of a tile; and the 32-row kernels that take the other widths."""
+import pytest
+import torch
+
+from oracle import moe_oracle as O
+from tolerances import assert_close
+
+pytestmark = pytest.mark.gpu
+
+# rows of successive experts: one row, the edges of a 16-row group, of a 32-row tile, several tiles
+EDGES = [1, 15, 16, 17, 31, 32, 33, 2, 47, 48, 49, 64, 65, 3]
+
+
+def _raw(pkg, lw, x, ids):
+    """experts() on given routing: its rows [T * 8, H] back in (token, slot) order."""
+    gr = pkg.abi.sort_permute(ids, lw.n_experts)
+    y = pkg.abi.experts(x, lw.gate_up_q, lw.gate_up_fmt, lw.down_q, lw.down_fmt, gr, 8,
+                        pkg._lib.MOE_PATH_MFMA, up_q=lw.up_q)
+    torch.cuda.synchronize()
+    return y.cpu()[gr["pair_pos"].cpu().long()]
+
+
+def _ids(T, counts, n_experts, seed):
+    """[T, 8] ids in which experts 3, 3 + 7, ... get the given row counts (the last takes the rest)."""
+    p = T * 8
+    flat = torch.cat([torch.full((n,), (3 + 7 * i) % n_experts, dtype=torch.int32) for i, n in enumerate(counts)])
+    assert flat.numel() <= p
+    rest = torch.arange(p - flat.numel(), dtype=torch.int32) % 2 + 1
+    flat = torch.cat([flat, rest])
+    return flat[torch.randperm(p, generator=torch.Generator().manual_seed(seed))].view(T, 8)
+
+
+def _rel(got, want):
+    return float((got.double() - want.double()).norm() / want.double().norm())
+
+
+# up to 256 tokens 16-row tiles, above 32-row ones; x and the SiLU rows are rounded to f16 (2^-11 / sqrt(12)
+# = 1.4e-4 rms each, three of them in a row: 2.4e-4), the weights not at all: 5e-4 is twice that
+@pytest.mark.parametrize("fixture,T", [("layer_c0", 64), ("layer_c0", 257), ("layer_q5k", 64),
+                                       ("layer_q5k", 257), ("layer_artifact", 100)])
+def test_rows_at_tile_edges(pkg, dev, request, fixture, T):
+    lw, ow = request.getfixturevalue(fixture)
+    x = pkg.synth.make_input(T, seed=T, device=dev)
+    ids = _ids(T, EDGES, lw.n_experts, T)
+    raw = _raw(pkg, lw, x, ids.to(dev))
+    sample = torch.randperm(T, generator=torch.Generator().manual_seed(T))[:48]
+    want = O.experts_and_combine(x.cpu()[sample], ids[sample].long(),
+                                 torch.ones(len(sample), 8, dtype=torch.bfloat16), ow)["expert_raw"]
+    got = raw.view(T, 8, -1)[sample]
+    assert_close(got, want, f"{fixture} T={T}")
+    assert _rel(got, want) <= 5e-4
+
+
+def test_one_tile_height_or_the_other_same_bits(pkg, layer_q5k, dev):
+    """A row's sums do not depend on the tile it sits in: 256 tokens (16-row tiles) and the same
+    tokens among 257 (32-row tiles), Q4_K gate_up and Q5_K down."""
+    lw, _ = layer_q5k
+    x = pkg.synth.make_input(257, seed=5, device=dev)
+    ids = _ids(257, EDGES, lw.n_experts, 6).to(dev)
+    a = _raw(pkg, lw, x[:256].contiguous(), ids[:256].contiguous())
+    b = _raw(pkg, lw, x, ids)[: 256 * 8]
+    assert torch.isfinite(a).all() and torch.equal(a, b)
+
+
+def test_large_and_small_activations(pkg, layer_c0, dev):
+    """Rows whose sub-block sums pass 65504 (their SiLU rows saturate, here as on the other tiles), and
+    small rows: x 0.05 gives SiLU rows of (0.05 0.9)^2 / 2 = 1e-3, still above f16's subnormals
+    (6e-5), so the bound of two roundings holds."""
+    lw, ow = layer_c0
+    x = pkg.synth.make_input(16, seed=9, device=dev)
+    x[:8] *= 8000.0
+    x[8:] *= 0.05
+    ids = _ids(16, [1, 17, 20], lw.n_experts, 9)
+    raw = _raw(pkg, lw, x, ids.to(dev)).view(16, 8, -1)
+    want = O.experts_and_combine(x.cpu(), ids.long(), torch.ones(16, 8, dtype=torch.bfloat16), ow)["expert_raw"]
+    assert torch.isfinite(raw).all()
+    assert _rel(raw[8:], want[8:]) <= 5e-4
+
+
+def test_other_widths_on_the_32_row_kernels(pkg, dev):
+    """hidden 4096: the few-rows kernels of the other widths, against the 160-row ones (whose K order
+    they share): the rows of a 256-token call equal those of the same tokens among 257."""
+    lw = pkg.synth.make_layer(seed=11, device=dev, n_experts=16, hidden=4096)
+    x = pkg.synth.make_input(257, seed=12, device=dev, hidden=4096)
+    ids = _ids(257, EDGES[:12], 16, 13).to(dev)
+    a = _raw(pkg, lw, x[:256].contiguous(), ids[:256].contiguous())
+    b = _raw(pkg, lw, x, ids)[: 256 * 8]
+    assert torch.isfinite(a).all() and torch.equal(a, b)

@@ -215,4 +215,28 @@ __device__ __forceinline__ float dot8_shared(const void* w, size_t row, int cols
   return dot8_bf16(*reinterpret_cast<const uint4*>(reinterpret_cast<const uint16_t*>(w) + row * cols + e0), x);
 }
 
+// the same eight weights held for several dots (dot8_shared's arithmetic)
+template <int SFMT>
+struct Row8 {
+  uint4 w;      // bf16 pairs, or (Q8_0) d's bits and the two words of quants
+};
+template <int SFMT>
+__device__ __forceinline__ Row8<SFMT> load_row8(const void* w, size_t row, int cols, int e0) {
+  Row8<SFMT> r;
+  if constexpr (SFMT == MOE_FMT_Q8_0) {
+    float d;
+    uint32_t lo, hi;
+    q8_0_load8(reinterpret_cast<const uint8_t*>(w) + row * (size_t)(cols / 32 * 34), e0, d, lo, hi);
+    r.w = make_uint4(__float_as_uint(d), lo, hi, 0u);
+  } else {
+    r.w = *reinterpret_cast<const uint4*>(reinterpret_cast<const uint16_t*>(w) + row * cols + e0);
+  }
+  return r;
+}
+template <int SFMT>
+__device__ __forceinline__ float dot_row8(const Row8<SFMT>& r, const float* x) {
+  if constexpr (SFMT == MOE_FMT_Q8_0) return q8_0_dot8(__uint_as_float(r.w.x), r.w.y, r.w.z, x);
+  else return dot8_bf16(r.w, x);
+}
+
 }  // namespace moe

@@ -87,3 +87,18 @@ def test_other_widths_on_the_32_row_kernels(pkg, dev):
     a = _raw(pkg, lw, x[:256].contiguous(), ids[:256].contiguous())
     b = _raw(pkg, lw, x, ids)[: 256 * 8]
     assert torch.isfinite(a).all() and torch.equal(a, b)
+
+
+@pytest.mark.parametrize("fixture", ["layer_c0", "layer_artifact"])
+@pytest.mark.parametrize("T", [2, 3, 5, 16])
+def test_shared_gemv_token_groups_same_bits(pkg, dev, request, fixture, T):
+    """Up to 16 tokens the shared expert runs as f32 dots over groups of one, two or four tokens: each
+    token's row and gate are those of a call of its own, bit for bit."""
+    lw, _ = request.getfixturevalue(fixture)
+    args = (lw.shared_gate, lw.shared_up, lw.shared_down, lw.shared_scalar_gate)
+    x = pkg.synth.make_input(T, seed=300 + T, device=dev)
+    raw, prob = pkg.abi.shared_expert(x, *args)
+    one = [pkg.abi.shared_expert(x[t:t + 1].contiguous(), *args) for t in range(T)]
+    torch.cuda.synchronize()
+    assert torch.equal(raw, torch.cat([r for r, _ in one]))
+    assert torch.equal(prob, torch.cat([p for _, p in one]))

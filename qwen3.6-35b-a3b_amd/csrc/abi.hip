@@ -417,6 +417,17 @@ static bool shared_skinny(int path, int sfmt, int T, int H, int Is) {
          moe_gemm5s_supports(H, Is);
 }
 
+// Q8_0 shared weights on narrow tiles (shared_q8.hip) up to this many tokens; above it the 160-row kernels,
+// which fetch and decode each weight once per 160 rows. Beside the router on the second stream the block
+// (artifact widths) took 221 against 248 us at 512 bf16 rows, 279 / 296 at 850, 301 / 303 at 1000; with f32
+// rows and the norm 243 / 253 at 512, 299 / 303 at 850, 327 / 314 at 1000.
+constexpr int kSharedQ8MaxT = 896;
+static bool shared_q8_tiles(int path, int sfmt, int T, int H, int Is) {
+  path = shared_path(path, T);
+  return (path == MOE_PATH_MFMA || path == MOE_PATH_MFMA_BF16) && sfmt == MOE_FMT_Q8_0 && T <= kSharedQ8MaxT &&
+         moe_sq8_supports(H, Is);
+}
+
 // x16: the f16 rows of x when the caller already has them (else NULL); x16_make: where to write
 // them for the caller (NULL: not wanted), made by the shared expert's own kernels where they can
 static int shared_body(const void* x, int x_dtype, const uint16_t* x16, const void* wg,
@@ -435,6 +446,11 @@ static int shared_body(const void* x, int x_dtype, const uint16_t* x16, const vo
     MOE_TRY(moe_launch_gemm5s_gateup(x, x_dtype, wg, wu, wsg, gate_dtype, T, H, Is, s, gate_prob, x16_make, st));
     made = x16_make != nullptr;
     return moe_launch_gemm5s_down(s, wd, T, H, Is, shared_raw, st);
+  }
+  if (shared_q8_tiles(path, sfmt, T, H, Is)) {
+    MOE_TRY(moe_launch_sq8_gateup(x, x_dtype, wg, wu, wsg, gate_dtype, T, H, Is, s, gate_prob, x16_make, st));
+    made = x16_make != nullptr;
+    return moe_launch_sq8_down(s, wd, T, H, Is, shared_raw, st);
   }
   // bf16 shared weights on the MFMA path: the dense 128-row kernels, on bf16 rows as they are.
   // With bf16 rows the GEMMs go first and the gate kernel last; it reads every row anyway and
@@ -641,22 +657,24 @@ static int block_forward_impl(const void* x, int x_dtype, int T, int H, int I, i
   // with bf16 rows and the shared expert forked, the shared GEMMs read the rows as they are and
   // the conversion runs on the shared expert's stream after them (off the router's path)
   const bool fork = T >= kForkMinT && allow_fork;
-  // Few rows per expert (the 32-row routed kernels) with the narrow-slab shared expert: no second
+  // Few rows per expert with the narrow-slab shared expert (bf16, or Q8_0 from 17 tokens on): no second
   // stream. The single-launch router also writes the f16 copy of x and runs the shared gate/up
   // blocks, and the shared down blocks run inside the routed down launch: both grids leave CUs
   // idle at this size, and the fork and join cost more than the shared expert's time left after
   // that overlap.
-  const bool fuse = rpath == MOE_PATH_MFMA && Wt.shared_fmt == MOE_FMT_BF16 && H % 2048 == 0 && I_s % 256 == 0 &&
-                    (mfma_reg_rows(rpath, T, H, I, gate_up_fmt, down_fmt) || mfma_small(rpath, T, H, I, gate_up_fmt, down_fmt)) &&
-                    shared_skinny(path, Wt.shared_fmt, T, H, I_s) && moe_router_chain_supported(T, H, E, K);
+  const int reg_rows = mfma_reg_rows(rpath, T, H, I, gate_up_fmt, down_fmt);
+  const bool sh_bf16 = shared_skinny(path, Wt.shared_fmt, T, H, I_s);
+  const bool sh_q8 = shared_q8_tiles(path, Wt.shared_fmt, T, H, I_s);
+  const bool fuse = rpath == MOE_PATH_MFMA && H % 2048 == 0 && I_s % 256 == 0 && T <= kSharedSkinnyMaxT &&
+                    (reg_rows ? sh_bf16 || sh_q8 : sh_bf16 && mfma_small(rpath, T, H, I, gate_up_fmt, down_fmt)) &&
+                    moe_router_chain_supported(T, H, E, K);
   uint16_t* x16 = nullptr;
   bool x16_late = false;
   if (rpath == MOE_PATH_MFMA) {
     x16 = reinterpret_cast<uint16_t*>(w.take((size_t)T * H * 2));
     if (!x16) return moe_set_error(MOE_E_WORKSPACE, "moe_block_forward: workspace too small");
     // made on the shared expert's stream: beside (or after) its GEMMs, off the router's path
-    x16_late = !fuse && fork && Wt.shared_fmt == MOE_FMT_BF16 &&
-               (x_dtype == MOE_DT_BF16 || shared_skinny(path, Wt.shared_fmt, T, H, I_s));
+    x16_late = !fuse && fork && (sh_q8 || (Wt.shared_fmt == MOE_FMT_BF16 && (x_dtype == MOE_DT_BF16 || sh_bf16)));
     if (!x16_late && !fuse) MOE_TRY(moe_launch_to_f16(x, x_dtype, (size_t)T * H, x16, st));
   }
   if (fuse) {
@@ -670,10 +688,10 @@ static int block_forward_impl(const void* x, int x_dtype, int T, int H, int I, i
     MoeShJob g, d;
     g.n = moe_shjob_gateup_blocks(T, I_s);
     g.x = x; g.x_dtype = x_dtype; g.wsg = ws_scalar_gate; g.gdt = Wt.scalar_gate_dtype;
-    g.gate_prob = gp; g.w0 = reinterpret_cast<const uint16_t*>(ws_gate);
-    g.w1 = reinterpret_cast<const uint16_t*>(ws_up); g.S = ssh; g.T = T; g.H = H; g.Is = I_s;
+    g.fmt = d.fmt = Wt.shared_fmt;
+    g.gate_prob = gp; g.w0 = ws_gate; g.w1 = ws_up; g.S = ssh; g.T = T; g.H = H; g.Is = I_s;
     d.n = moe_shjob_down_blocks(T, H);
-    d.w0 = reinterpret_cast<const uint16_t*>(ws_down); d.S = ssh; d.y = sraw; d.T = T; d.H = H; d.Is = I_s;
+    d.w0 = ws_down; d.S = ssh; d.y = sraw; d.T = T; d.H = H; d.Is = I_s;
     // the sort and the tile list inside the router launch, by its last group to finish routing
     MoeSortJob sj;
     if (tiles && bm >= MOE_GEMM8_BM && bm <= 160) {

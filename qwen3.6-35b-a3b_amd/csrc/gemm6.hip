@@ -227,7 +227,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   if ((int)blockIdx.x >= nr) {
     // the small-T shared expert's down: y = shared_raw
     const int b = (int)blockIdx.x - nr, nslab = sh.H / 32;
-    shs::down_tile<4, 32>(sh.S, sh.w0, sh.T, sh.H, sh.Is, b % nslab, (b / nslab) * 32, sh.y,
+    shs::down_tile<4, 32>(sh.S, reinterpret_cast<const uint16_t*>(sh.w0), sh.T, sh.H, sh.Is, b % nslab, (b / nslab) * 32, sh.y,
                           reinterpret_cast<float*>(&sm));
     return;
   }
@@ -294,8 +294,8 @@ static dim3 g6_grid(int max_tiles, int ncol) {
 // over 4 waves in 64-wide chunks)
 static int check_shjob(const MoeShJob* sh) {
   if (!sh || sh->n == 0) return MOE_OK;
-  if (sh->H % 32 || sh->Is % 256 || !sh->S || !sh->w0 || !sh->y)
-    return moe_set_error(MOE_E_UNSUPPORTED, "gemm6: shared-expert blocks need H %% 32 == 0, I_s %% 256 == 0 and every pointer");
+  if (sh->H % 32 || sh->Is % 256 || sh->fmt != MOE_FMT_BF16 || !sh->S || !sh->w0 || !sh->y)
+    return moe_set_error(MOE_E_UNSUPPORTED, "gemm6: shared-expert blocks need bf16 weights, H %% 32 == 0, I_s %% 256 == 0 and every pointer");
   const int want = moe_shjob_down_blocks(sh->T, sh->H);
   if (sh->n != want) return moe_set_error(MOE_E_ARG, "gemm6: %d shared-expert blocks given, %d needed", sh->n, want);
   return MOE_OK;

@@ -523,8 +523,13 @@ __global__ __launch_bounds__(64 * g8::kDnWaves, (RMAX == 1 ? 4 : 3)) void k_gemm
   if ((int)blockIdx.x >= nr) {
     // the small-T shared expert's down: y = shared_raw
     const int b = (int)blockIdx.x - nr, nslab = sh.H / 32;
-    shs::down_tile<4, 32>(sh.S, sh.w0, sh.T, sh.H, sh.Is, b % nslab, (b / nslab) * 32, sh.y,
-                          reinterpret_cast<float*>(g8_lds));
+    float* red = reinterpret_cast<float*>(g8_lds);
+    if (sh.fmt == MOE_FMT_Q8_0)
+      shs::down_tile_q8<kDnWaves>(sh.S, reinterpret_cast<const uint8_t*>(sh.w0), sh.T, sh.H, sh.Is, b % nslab,
+                                  (b / nslab) * 32, sh.y, red);
+    else
+      shs::down_tile<kDnWaves, 32>(sh.S, reinterpret_cast<const uint16_t*>(sh.w0), sh.T, sh.H, sh.Is, b % nslab,
+                                   (b / nslab) * 32, sh.y, red);
     return;
   }
   Item it;

@@ -108,6 +108,13 @@ int moe_launch_gemm5s_gateup(const void* x, int x_dtype, const void* w_gate, con
 int moe_launch_gemm5s_down(const uint16_t* S, const void* w_down, int T, int H, int Is, float* y,
                            hipStream_t st);
 
+// shared_q8.hip: the same for Q8_0 weights (32-row token tiles); x in its own dtype
+bool moe_sq8_supports(int H, int Is);
+int moe_launch_sq8_gateup(const void* x, int x_dtype, const void* w_gate, const void* w_up, const void* wsg,
+                          int gate_dtype, int T, int H, int Is, uint16_t* S, float* gate_prob, uint16_t* x16,
+                          hipStream_t st);
+int moe_launch_sq8_down(const uint16_t* S, const void* w_down, int T, int H, int Is, float* y, hipStream_t st);
+
 // gemm4.hip: Q4_K gate_up and down with the weight decode in the MFMA waves (persistent grid,
 // direct global->LDS operand loads, two blocks per CU); same tiles (MOE_GEMM3_BM rows),
 // arguments and results as the gemm3 launchers for Q4_K, within f32 rounding (another k order).
@@ -137,8 +144,9 @@ struct MoeShJob {
   const void* wsg = nullptr;       // the scalar gate's row and its dtype
   int gdt = 0;
   float* gate_prob = nullptr;
-  const uint16_t* w0 = nullptr;    // gate/up: w_gate [Is, H]; down: w_down [H, Is]
-  const uint16_t* w1 = nullptr;    // gate/up: w_up [Is, H]
+  int fmt = MOE_FMT_BF16;          // or MOE_FMT_Q8_0
+  const void* w0 = nullptr;        // gate/up: w_gate [Is, H]; down: w_down [H, Is]
+  const void* w1 = nullptr;        // gate/up: w_up [Is, H]
   uint16_t* S = nullptr;           // gate/up: written; down: read (f16 [T, Is])
   float* y = nullptr;              // down: shared_raw (f32 [T, H])
   int T = 0, H = 0, Is = 0;

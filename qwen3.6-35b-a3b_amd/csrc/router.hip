@@ -807,7 +807,12 @@ __global__ __launch_bounds__(512) void k_router_chain(
     // the small-T shared expert's gate/up tile (32 token rows x 16 columns), x read as it is,
     // then the scalar gate of this block's share of the tokens
     const int b = (int)blockIdx.x - nr, nslab = sh.Is / 16;
-    shs::gateup_tile<XDT, 8, 32>(xv, sh.w0, sh.w1, T, H, sh.Is, b % nslab, (b / nslab) * 32, sh.S, sm.red);
+    if (sh.fmt == MOE_FMT_Q8_0)
+      shs::gateup_tile_q8<XDT, 8>(xv, reinterpret_cast<const uint8_t*>(sh.w0), reinterpret_cast<const uint8_t*>(sh.w1),
+                                  T, H, sh.Is, b % nslab, (b / nslab) * 32, sh.S, sm.red);
+    else
+      shs::gateup_tile<XDT, 8, 32>(xv, reinterpret_cast<const uint16_t*>(sh.w0), reinterpret_cast<const uint16_t*>(sh.w1),
+                                   T, H, sh.Is, b % nslab, (b / nslab) * 32, sh.S, sm.red);
     shs::gate_rows<XDT>(xv, sh.wsg, sh.gdt, T, H, sh.gate_prob, b * 8 + wv, sh.n * 8);
     return;
   }

@@ -4,7 +4,7 @@
 // 32-row groups for its range in registers (no LDS staging: every operand is used once per block);
 // the NW f32 partial tiles meet in LDS and are added in wave order before the epilogue (gate/up:
 // SiLU(gate) * up to f16, a slab = 16 gate + the matching 16 up rows in one 32-column MFMA group;
-// down: f32 rows, a slab = 32 rows of w_down).
+// down: f32 rows, a slab = 32 rows of w_down). The Q8_0 forms take 32-row token tiles.
 #pragma once
 #include "common.h"
 #include "gemv_dev.h"
@@ -198,6 +198,120 @@ __device__ __forceinline__ void down_tile(const uint16_t* S, const uint16_t* wd,
       v.w = red_sum<NW>(red, rr, c + 3);
       *reinterpret_cast<float4*>(y + (size_t)(m0 + rr) * H + 32 * slab + c) = v;
     }
+  }
+}
+
+// ---- the same tiles with Q8_0 weights: 32 token rows, v_mfma_f32_16x16x32_f16, one MFMA per 32-element
+// block and 16 x 16 outputs, the quants as exact f16 whole numbers and the block's d applied to the
+// sum in f32 (f16(x), as the 160-row kernels take it; the weights are not rounded). Lane (m, g) =
+// (l % 16, l / 16) holds token row m / weight row m and elements 8 g .. 8 g + 7 of the block.
+typedef _Float16 h2_t __attribute__((ext_vector_type(2)));
+typedef float f32x4_t __attribute__((ext_vector_type(4)));
+
+__device__ __forceinline__ uint4 q8_frag(uint32_t lo, uint32_t hi) {
+  // q + 128 under the f16 exponent of 1024, less 1152
+  auto pair = [](uint32_t w, uint32_t sel) {
+    return __builtin_bit_cast(uint32_t, __builtin_bit_cast(h2_t, __builtin_amdgcn_perm(0x64646464u, w, sel)) -
+                                            (h2_t){(_Float16)1152.0f, (_Float16)1152.0f});
+  };
+  lo ^= 0x80808080u;
+  hi ^= 0x80808080u;
+  return make_uint4(pair(lo, 0x04010400u), pair(lo, 0x04030402u), pair(hi, 0x04010400u), pair(hi, 0x04030402u));
+}
+template <int AT>
+__device__ __forceinline__ uint4 a_frag_f16(const ARaw<AT>& r) {
+  if constexpr (AT == MOE_DT_BF16)
+    return make_uint4(f16x2_sat(bf16_to_f32(r.v[0].x & 0xFFFFu), bf16_to_f32(r.v[0].x >> 16)),
+                      f16x2_sat(bf16_to_f32(r.v[0].y & 0xFFFFu), bf16_to_f32(r.v[0].y >> 16)),
+                      f16x2_sat(bf16_to_f32(r.v[0].z & 0xFFFFu), bf16_to_f32(r.v[0].z >> 16)),
+                      f16x2_sat(bf16_to_f32(r.v[0].w & 0xFFFFu), bf16_to_f32(r.v[0].w >> 16)));
+  else
+    return a_frag<AT>(r);
+}
+
+// The block's partial tiles: rows m0 .. m0 + 16 RG - 1 of a (type AT, K wide) times weight rows w0 + m
+// (column group 0) and w1 + m (group 1), K split over the waves; [wave][row group][column
+// group][lane] of four floats (row 4 g + i of the group).
+template <int AT, int NW, int RG>
+__device__ __forceinline__ void tile_q8(const void* a, int T, int K, int m0, const uint8_t* w0, const uint8_t* w1,
+                                        float* red) {
+  const int lane = threadIdx.x & 63, m = lane & 15, g = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  constexpr int es = AT == MOE_DT_F32 ? 4 : 2;
+  const size_t rowb = (size_t)(K / 32) * 34;
+  const int k0 = wave * (K / NW) + 8 * g, nb = K / NW / 32;
+  const uint8_t* ab = reinterpret_cast<const uint8_t*>(a);
+  const uint8_t* ar[RG];
+#pragma unroll
+  for (int r = 0; r < RG; ++r) ar[r] = ab + ((size_t)min(m0 + 16 * r + m, T - 1) * K + k0) * es;
+  const uint8_t *b0 = w0 + m * rowb, *b1 = w1 + m * rowb;
+  f32x4_t acc[RG][2] = {};
+#pragma unroll 4
+  for (int b = 0; b < nb; ++b) {
+    ARaw<AT> x[RG];
+#pragma unroll
+    for (int r = 0; r < RG; ++r) ld_a<AT>(x[r], ar[r] + b * 32 * es);
+    float d[2];
+    uint32_t lo[2], hi[2];
+    q8_0_load8(b0, k0 + 32 * b, d[0], lo[0], hi[0]);
+    q8_0_load8(b1, k0 + 32 * b, d[1], lo[1], hi[1]);
+    const f16x8_t w[2] = {__builtin_bit_cast(f16x8_t, q8_frag(lo[0], hi[0])), __builtin_bit_cast(f16x8_t, q8_frag(lo[1], hi[1]))};
+#pragma unroll
+    for (int r = 0; r < RG; ++r) {
+      const f16x8_t av = __builtin_bit_cast(f16x8_t, a_frag_f16<AT>(x[r]));
+#pragma unroll
+      for (int c = 0; c < 2; ++c) {
+        const f32x4_t v = __builtin_amdgcn_mfma_f32_16x16x32_f16(av, w[c], (f32x4_t){}, 0, 0, 0);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) acc[r][c][i] = fmaf(d[c], v[i], acc[r][c][i]);
+      }
+    }
+  }
+#pragma unroll
+  for (int r = 0; r < RG; ++r)
+#pragma unroll
+    for (int c = 0; c < 2; ++c)
+      *reinterpret_cast<f32x4_t*>(red + (((wave * RG + r) * 2 + c) * 64 + lane) * 4) = acc[r][c];
+  __syncthreads();
+}
+// LDS floats of the partial tiles
+template <int NW, int RG>
+constexpr int red_q8_floats() { return NW * RG * 512; }
+// sum over the waves (in wave order) of tile row rr, column group c, column n
+template <int NW, int RG>
+__device__ __forceinline__ float red_q8(const float* red, int rr, int c, int n) {
+  const float* p = red + ((2 * (rr >> 4) + c) * 64 + n + 16 * ((rr & 15) >> 2)) * 4 + (rr & 3);
+  float s = p[0];
+#pragma unroll
+  for (int w = 1; w < NW; ++w) s += p[w * RG * 512];
+  return s;
+}
+// S rows m0 .. m0 + 16 RG - 1 (< T), columns 16 slab .. + 15 (f16) = SiLU(a wg^T) * (a wu^T)
+template <int AT, int NW, int RG = 2>
+__device__ __forceinline__ void gateup_tile_q8(const void* a, const uint8_t* wg, const uint8_t* wu, int T, int H, int Is,
+                                               int slab, int m0, uint16_t* __restrict__ S, float* red) {
+  const size_t r0 = (size_t)(16 * slab) * (H / 32 * 34);
+  tile_q8<AT, NW, RG>(a, T, H, m0, wg + r0, wu + r0, red);
+  for (int o = threadIdx.x; o < 16 * RG * 16; o += NW * 64) {
+    const int rr = o >> 4, n = o & 15;
+    if (m0 + rr < T) {
+      const float gv = red_q8<NW, RG>(red, rr, 0, n), uv = red_q8<NW, RG>(red, rr, 1, n);
+      float v = gv * __builtin_amdgcn_rcpf(1.0f + __expf(-gv)) * uv;
+      v = fminf(fmaxf(v, -65504.0f), 65504.0f);
+      S[(size_t)(m0 + rr) * Is + 16 * slab + n] = __builtin_bit_cast(uint16_t, (_Float16)v);
+    }
+  }
+}
+// y rows m0 .. m0 + 16 RG - 1 (< T), columns 32 slab .. + 31 (f32) = S wd^T
+template <int NW, int RG = 2>
+__device__ __forceinline__ void down_tile_q8(const uint16_t* S, const uint8_t* wd, int T, int H, int Is, int slab,
+                                             int m0, float* __restrict__ y, float* red) {
+  const size_t rowb = (size_t)(Is / 32) * 34;
+  const uint8_t* w = wd + (size_t)(32 * slab) * rowb;
+  tile_q8<kF16, NW, RG>(S, T, Is, m0, w, w + 16 * rowb, red);
+  for (int o = threadIdx.x; o < 16 * RG * 32; o += NW * 64) {
+    const int rr = o >> 5, n = o & 31;
+    if (m0 + rr < T) y[(size_t)(m0 + rr) * H + 32 * slab + n] = red_q8<NW, RG>(red, rr, n >> 4, n & 15);
   }
 }
 

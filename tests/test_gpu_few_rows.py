@@ -102,3 +102,22 @@ def test_shared_gemv_token_groups_same_bits(pkg, dev, request, fixture, T):
     torch.cuda.synchronize()
     assert torch.equal(raw, torch.cat([r for r, _ in one]))
     assert torch.equal(prob, torch.cat([p for _, p in one]))
+
+
+# 32-row token tiles up to 256 tokens, 64-row tiles to 896, the 160-row kernels above; x and the SiLU rows
+# are rounded to f16, the quants are exact (the bound of the routed rows above)
+@pytest.mark.parametrize("T,dtype", [(17, torch.float32), (32, torch.bfloat16), (33, torch.float32),
+                                     (257, torch.bfloat16), (321, torch.float32), (896, torch.bfloat16),
+                                     (897, torch.float32)])
+def test_q8_0_shared_tiles(pkg, layer_artifact, dev, T, dtype):
+    lw, ow = layer_artifact
+    x = pkg.synth.make_input(T, seed=400 + T, device=dev, dtype=dtype)
+    raw, prob = pkg.abi.shared_expert(x, lw.shared_gate, lw.shared_up, lw.shared_down, lw.shared_scalar_gate)
+    torch.cuda.synchronize()
+    rows = torch.cat([torch.arange(min(T, 40)), torch.tensor([T - 2, T - 1])])
+    want = O.shared_expert(x.cpu()[rows], ow)
+    assert torch.isfinite(raw).all()
+    assert_close(raw.cpu()[rows], want["shared_raw"], f"T={T}")
+    if T <= 896:
+        assert _rel(raw.cpu()[rows], want["shared_raw"]) <= 5e-4
+    assert torch.allclose(prob.cpu()[rows], want["shared_gate_prob"].view(-1), rtol=1e-5, atol=1e-6)

@@ -22,6 +22,11 @@ __device__ __forceinline__ void load16(uint32_t off, const void* base, uint32_t 
                : "memory");
 }
 
+// 16 bytes per lane from the lane's own address
+__device__ __forceinline__ void load16(const void* p, uint32_t lds) {
+  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(p), "s"(lds) : "memory");
+}
+
 // s_waitcnt vmcnt(n), other counters untouched (gfx9 encoding: vmcnt bits 3:0 and 15:14)
 template <int N>
 __device__ __forceinline__ void wait_vm() {

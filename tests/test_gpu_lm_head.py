@@ -98,3 +98,44 @@ def test_lm_head_refusals(pkg, dev):
         pkg.abi.lm_head(h, t, pkg._lib.MOE_FMT_Q6_K)                  # B > 8
     with pytest.raises(pkg.abi.Refused):
         pkg.abi.lm_head(h[:1], t, pkg._lib.MOE_FMT_Q4_K)              # not a table format
+
+
+@pytest.mark.parametrize("fmt_name", ["Q6_K", "Q8_0"])
+@pytest.mark.parametrize("B,hdt", [(2, torch.float32), (4, torch.bfloat16), (5, torch.float32), (8, torch.float32)])
+@pytest.mark.parametrize("n", [1, 15, 17, 9001])       # around 16 rows an iteration; several iterations per block
+def test_lm_head_int8_digits(pkg, dev, fmt_name, B, hdt, n):
+    """Two or more tokens: fixed-point digits under each 256-element slice's largest value. Error bound per
+    output: 16 f32 roundings of sums no larger than sum |h w|, and what 30 bits under the slice's maximum
+    and the lower digits' roundings (digits up to 2^-7 of the maximum) leave: 2^-26 max |h| sum |w| a slice."""
+    fmt = getattr(pkg._lib, "MOE_FMT_" + fmt_name)
+    V = max(n, 64)
+    t, dec = _table(pkg, fmt, V, seed=41)
+    g = torch.Generator().manual_seed(42 + B)
+    h = torch.randn(B, H, generator=g)
+    h[0, 5], h[0, 300:556] = 3.0e4, 0.0                 # one large value, a slice of zeros
+    h[1] *= 1e-30
+    if B > 3:
+        h[2] *= 1e30
+        h[3, 77] = float("inf")
+    if B > 4:
+        h[4, 2047] = float("nan")
+    h = h.to(hdt)
+    ids = torch.randint(0, V, (n,), generator=g, dtype=torch.int32)
+    ids[n // 2:n // 2 + 1] = V
+    rows = ids.numpy().copy()
+    rows[n // 2] = 0
+    for gather in (False, True):
+        got = pkg.abi.lm_head(h.to(dev), t.to(dev) if gather else t[:n].contiguous().to(dev), fmt,
+                              row_ids=ids.to(dev) if gather else None)
+        out, w = got.cpu().double().numpy(), dec[rows] if gather else dec[:n]
+        if gather:
+            assert np.isnan(out[:, n // 2]).all()
+            out, w = np.delete(out, n // 2, 1), np.delete(w, n // 2, 0)
+        hd, wd = h.double().numpy(), w.astype(np.float64)
+        for b in range(B):
+            if not np.isfinite(hd[b]).all():
+                assert np.isnan(out[b]).all()
+                continue
+            hs, ws = hd[b].reshape(8, 256), np.abs(wd).reshape(-1, 8, 256)
+            tol = 2.0 ** -20 * (np.abs(wd) @ np.abs(hd[b])) + 2.0 ** -26 * (ws.sum(2) @ np.abs(hs).max(1))
+            assert (np.abs(out[b] - wd @ hd[b]) <= tol).all(), (b, np.max(np.abs(out[b] - wd @ hd[b]) / tol))

@@ -7,8 +7,9 @@
  * moe_block_forward* call on a device that runs the shared expert beside the routed path creates
  * that device's second stream (default priority, non-blocking) and two events, kept until the
  * process ends. That is a call of 7 or more tokens, except where the step folds the shared expert
- * into its own launches (up to 256 tokens with Q4_K routed weights, bf16 shared weights,
- * H % 2048 == 0 and I_s % 256 == 0: one stream). moe_block_forward_w_noalloc never forks. Routing values never
+ * into its own launches (8 to 256 tokens with Q4_K gate_up, Q4_K down or, at H = 2048, Q5_K down,
+ * shared weights in bf16 or, at H = 2048 and from 17 tokens on, Q8_0, H % 2048 == 0 and
+ * I_s % 256 == 0: one stream). moe_block_forward_w_noalloc never forks. Routing values never
  * travel to the host (specification/11-moe-block.md §11.7: the block is computable with zero
  * host-visible routing values).
  *
@@ -257,8 +258,10 @@ int moe_block_forward_w_noalloc(const void *x, int x_dtype, int T, int H, int I,
  * id outside [0, V) gives NaN for that output). h: [B, H] f32 or bf16 (h_dtype); W: V rows of H
  * in w_fmt: MOE_FMT_Q6_K (H/256 x 210 B per row: the shipped artifact's output.weight,
  * engine/README.md:33), MOE_FMT_Q8_0 (H/32 x 34 B) or MOE_FMT_BF16 (H x 2 B); W 16-byte aligned.
- * logits: [B, n_rows] f32. Limits: H == 2048. Tokens go in passes of up to 4, each reading the
- * table once. Results are f32 dots in this kernel's association order: they lie within the
+ * logits: [B, n_rows] f32. Limits: H == 2048. The table is read once; a bf16 one once per 4
+ * tokens. Results are f32 dots in the kernel's association order, or (Q6_K, Q8_0, but for one token
+ * of a short row list) sums of exact integer products over h in fixed point, 30 bits under the largest
+ * value of each 256-element slice (a token with an infinity or NaN gives NaN): they lie within the
  * reference's band gamma_n * sum_k |h_k w_k| (n = K-1 for exact products, 2K-1 otherwise;
  * prototype/lm_head/gate.py:214-240) of the exact dot. Replaces prototype/lm_head/
  * lm_head_kernels.h:474-512 (lmh_dot_batch) as launched by prototype/lm_head/lm_head.hip:51. */
@@ -270,7 +273,7 @@ int moe_lm_head(const void *h, int h_dtype, int B, int H, const void *w, int w_f
  * bounded wait of the single-launch decode layer gave up (its workgroups were not all co-resident,
  * or not placed on the XCDs round robin as it assumes); the output rows of every workgroup that
  * gave up are NaN and the rest of that call's outputs are unspecified. Bit MOE_STATUS_SYNC_STATE:
- * a block-arrival counter of the single-launch router (8 to 256 tokens) held a count its launch
+ * a block-arrival counter of the single-launch router (2 to 256 tokens) held a count its launch
  * cannot produce (a workspace that skipped moe_workspace_init, or two calls overlapping on one
  * workspace); that call's logits, ids, weights and block outputs are unspecified (every stage of
  * the launch still runs once, so the grouped GEMMs after it stay in bounds), and

@@ -1,6 +1,8 @@
 // Prefill-path grouped GEMM for few rows per expert (small batches): Q4_K gate_up and down with
 // the weight decode in the MFMA waves (gfx950, v_mfma_f32_32x32x16_f16, f32 accumulation).
 //
+// Used for widths other than H = 2048: there gemm8.hip's kernels are faster (gate_up, 64 tokens, uniform
+// routing: 85 us here, 57 there).
 // When T * K / E is small an expert has a few dozen (token, slot) rows. The 160-row persistent
 // kernels (gemm4.hip) then run one short item per block and wait, at every K step, for that
 // step's activation rows, which they request one step ahead: the step time is an L2 round trip.

@@ -25,7 +25,7 @@ bool moe_router_i8_supported(int T, int H, int E);
 int moe_launch_router_logits_i8(const void* x, int x_dtype, const void* w, int w_dtype,
                                 const float* bias, int T, int H, int E, uint16_t* logits,
                                 void* scratch, hipStream_t st);
-// R1-R5 in one launch (8 <= T <= 256, E = 256, K = 8, H % 2048 == 0): scratch of
+// R1-R5 in one launch (2 <= T <= 256, E = 256, K = 8, H % 2048 == 0): scratch of
 // moe_router_chain_scratch_bytes(T, E) bytes, sync = the workspace's sync words (arrival counters
 // at kRouterCntWord, zero between launches). Same bits as router_logits + route_topk.
 bool moe_router_chain_supported(int T, int H, int E, int K);
@@ -136,7 +136,7 @@ int moe_launch_gemm7_down(const uint16_t* S, const void* w_down, size_t expert_s
                           void* y, int y16, hipStream_t st);
 
 // The small-T shared expert's blocks (shared_small.h), appended to another launch's grid: gate/up
-// (with the scalar gate) in the single-launch router's, down in the gemm6 down launch's.
+// (with the scalar gate) in the single-launch router's, down in the gemm6 or gemm8 down launch's.
 struct MoeShJob {
   int n = 0;                       // shared-expert blocks appended to the launch
   const void* x = nullptr;         // gate/up: x [T, H], read as it is

@@ -594,7 +594,7 @@ constexpr int kChainTiles = 256;  // tile counters (T <= 256, E = 256); 16 group
 constexpr int kChainSortCnt = kChainTiles + 16;   // then the count of groups routed (the fused sort)
 static_assert((kRouterCntWord + kChainSortCnt + 1) * 4 <= (int)kSyncBytes, "router counters in the sync words");
 
-// ------------------------------------------- R1-R5 in one launch, 8 <= T <= 256, E = 256, K = 8 --
+// ------------------------------------------- R1-R5 in one launch, 2 <= T <= 256, E = 256, K = 8 --
 // The small-T R1 above runs one 16 x 16 tile per block, so at T = 64 it keeps 64 CUs busy for the
 // whole K; here each tile's K is split over kChainKS blocks (grid = tiles x kChainKS: 256 blocks at
 // T = 64), and the launches of R2-R5 are folded in:
@@ -645,7 +645,7 @@ __device__ __forceinline__ void stores_done() {
 // The stable grouping of the P = T * 8 pairs by expert (E = 256) by one 512-thread block: the
 // positions of moe_launch_sort (pairs p = t * 8 + k ordered by expert, equal experts in ascending
 // p; a stable counting sort, so any correct one gives the same positions), the offsets, the hit
-// list, and the bm-row tile list in build_tiles_block's order (by decreasing 32-row group count,
+// list, and (tiles not NULL) the bm-row tile list in build_tiles_block's order (by decreasing 32-row group count,
 // then ascending expert; an expert's full tiles before its partial one). The ids come from other
 // blocks of the launch, so they are read by agent-scope loads. P <= 2048, bm <= 160.
 struct ChainSortLds {
@@ -731,16 +731,16 @@ __device__ void chain_sort(const int32_t* __restrict__ ids, const MoeSortJob& j,
       acc += field(tp0, tp1, g);
     }
     const int p_full = gstart[ngmax] + field(pre0, pre1, ngmax);
-    for (int i = 0; i < nfull; ++i) {
+    for (int i = 0; i < nfull && j.tiles; ++i) {
       j.tiles[1 + 2 * (p_full + i)] = e;
       j.tiles[2 + 2 * (p_full + i)] = base + i * j.bm;
     }
-    if (grem) {
+    if (grem && j.tiles) {
       const int pt = gstart[grem] + field(pre0, pre1, grem) + (grem == ngmax ? nfull : 0);
       j.tiles[1 + 2 * pt] = e;
       j.tiles[2 + 2 * pt] = base + nfull * j.bm;
     }
-    if (e == 0) j.tiles[0] = acc;
+    if (e == 0 && j.tiles) j.tiles[0] = acc;
   }
   // the scatter, 512 pairs a round: ranks inside a wave from id matching (8 ballots on the id
   // bits), across waves from per-wave counts, across rounds from run[]
@@ -1021,7 +1021,7 @@ static void launch_router_logits(const void* x, const void* w, const float* bias
 }
 
 bool moe_router_chain_supported(int T, int H, int E, int K) {
-  return T >= 8 && T <= 256 && E == 256 && K == 8 && H % (64 * 8 * kChainKS) == 0;
+  return T >= 2 && T <= 256 && E == 256 && K == 8 && H % (64 * 8 * kChainKS) == 0;
 }
 
 size_t moe_router_chain_scratch_bytes(int T, int E) {
@@ -1039,7 +1039,7 @@ int moe_launch_router_chain(const void* x, int x_dtype, const void* w, int w_dty
                             void* scratch, int* sync, hipStream_t st, uint16_t* x16,
                             const MoeShJob* sh, const MoeSortJob* srt) {
   if (!moe_router_chain_supported(T, H, E, 8) || !scratch || !sync)
-    return moe_set_error(MOE_E_UNSUPPORTED, "router_chain: needs 8 <= T <= 256, E = 256, K = 8, H %% 2048 == 0");
+    return moe_set_error(MOE_E_UNSUPPORTED, "router_chain: needs 2 <= T <= 256, E = 256, K = 8, H %% 2048 == 0");
   const MoeShJob job = sh ? *sh : MoeShJob{};
   if (job.n) {
     if (job.T != T || job.H != H || job.Is % 256 || !job.w0 || !job.w1 || !job.S || !job.wsg || !job.gate_prob)
@@ -1050,7 +1050,7 @@ int moe_launch_router_chain(const void* x, int x_dtype, const void* w, int w_dty
   }
   const MoeSortJob sj = srt ? *srt : MoeSortJob{};
   if (sj.P) {
-    if (sj.P != T * 8 || !sj.offsets || !sj.sorted || !sj.pos || !sj.hits || !sj.tiles || sj.bm < MOE_GEMM8_BM || sj.bm > 160)
+    if (sj.P != T * 8 || !sj.offsets || !sj.sorted || !sj.pos || !sj.hits || sj.bm < MOE_GEMM8_BM || sj.bm > 160)
       return moe_set_error(MOE_E_ARG, "router_chain: the fused sort needs P = 8 T, 16 <= bm <= 160 and every output");
   }
   dim3 grid(((T + 15) / 16) * (E / 16) * kChainKS);

@@ -1,5 +1,5 @@
 // The small-T shared expert's dense GEMM pieces (gemm5.hip's own launches, and the blocks the
-// routed small-T launches run for it, gemm6.hip): one block per (64-row token tile, narrow weight
+// routed small-T launches run for it, gemm6.hip and gemm8.hip): one block per (64-row token tile, narrow weight
 // slab), the block's NW waves splitting K into contiguous ranges, each wave holding the tile's two
 // 32-row groups for its range in registers (no LDS staging: every operand is used once per block);
 // the NW f32 partial tiles meet in LDS and are added in wave order before the epilogue (gate/up:

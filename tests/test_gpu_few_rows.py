@@ -121,3 +121,28 @@ def test_q8_0_shared_tiles(pkg, layer_artifact, dev, T, dtype):
     if T <= 896:
         assert _rel(raw.cpu()[rows], want["shared_raw"]) <= 5e-4
     assert torch.allclose(prob.cpu()[rows], want["shared_gate_prob"].view(-1), rtol=1e-5, atol=1e-6)
+
+
+@pytest.mark.parametrize("fixture", ["layer_c0", "layer_artifact"])
+@pytest.mark.parametrize("T", [2, 3, 6])
+@pytest.mark.parametrize("ties", [False, True])
+def test_few_tokens_routed_in_one_launch(pkg, dev, request, fixture, T, ties):
+    """2 to 6 tokens: logits, routing and sort of the block in one launch, bit for bit the router call's
+    logits, ids and weights (ties: every expert of two groups has the same row), twice on one workspace."""
+    import copy
+    lw, ow = request.getfixturevalue(fixture)
+    if ties:
+        lw, ow = copy.copy(lw), copy.copy(ow)
+        lw.router = lw.router.clone()
+        lw.router[40:60], lw.router[200:230] = lw.router[40].clone(), lw.router[200].clone()
+        lw.router_bias = None
+    x = pkg.synth.make_input(T, seed=500 + T, device=dev)
+    want = pkg.abi.router_topk(x, lw.router, 8, bias=lw.router_bias)
+    for _ in range(2):
+        got = pkg.abi.block_forward(x, lw, stages=True)
+        torch.cuda.synchronize()
+        for k in ("router_logits", "topk_ids", "topk_weights"):
+            assert torch.equal(got[k].view(want[k].shape), want[k]), k
+        if not ties:
+            assert_close(got["combined_out"].cpu(), O.moe_block(x.cpu(), ow)["combined_out"], f"T={T}")
+    assert pkg.abi.device_error_bits(dev) == 0

@@ -243,6 +243,14 @@ __device__ __forceinline__ void zero_pads(uint8_t* sm, int slots) {
     *reinterpret_cast<uint32_t*>(sm + i / (4 * R) * slot_bytes<R>() + R * kFrag + (i / 4 % R) * kSum + 512 + 4 * (i & 3)) = 0u;
 }
 
+// A list of at most kFewTiles 16-row tiles (skewed routing, or a dozen tokens) leaves most CUs one block or
+// none: its tiles are cut into kGuFine (gate_up) and kDnFine (down) times the slabs, the same sums. The count
+// is known on the device only, so the kernels choose. Block us, coarse -> fine, Zipf routing: 64 tokens (66 tiles)
+// 72.6 -> 66.1, 32 (43) 59.2 -> 54.9, 16 (28) 69.8 -> 60.6. At 96 tiles (16 tokens, uniform) even twice the slabs
+// lose: 88 -> 91.
+constexpr int kFewTiles = 80, kGuFine = 4, kDnFine = 2;
+__device__ __forceinline__ bool few_tiles(const int32_t* __restrict__ tiles) { return tiles[0] <= kFewTiles; }
+
 struct Item {
   int e, m0, rows, col;
 };
@@ -409,13 +417,13 @@ __device__ __forceinline__ void gateup_item(const Item& it, const uint16_t* __re
   }
 }
 
-// ---- down: 512 columns per block, four passes of 128, wave w: 32 of each -----------------------
+// ---- down: 512 columns per block (few tiles: 256), passes of 128, wave w: 32 of each -------------
 // The tile's whole rows (I of K) sit in LDS, staged once.
 constexpr int kDownCols = 512, kPassCols = 32 * kDnWaves;
 template <int R, int FMT, bool Y16>
 __device__ __forceinline__ void down_item(const Item& it, const uint16_t* __restrict__ S,
                                           const uint8_t* __restrict__ wd, size_t estride, int H, int I,
-                                          void* __restrict__ y, uint8_t* sm) {
+                                          int cols, void* __restrict__ y, uint8_t* sm) {
   const int t = threadIdx.x, lane = t & 63, m = lane & 15, g = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
   const int nsb = I / 256;
@@ -425,9 +433,9 @@ __device__ __forceinline__ void down_item(const Item& it, const uint16_t* __rest
 #pragma unroll
   for (int p = 0; p < 2 * R; ++p)
     roff[p] = (uint32_t)min((t >> 5) + 8 * p, it.rows - 1) * (uint32_t)I * 2u + 16u * (t & 31);
-  // pass cb: columns it.col 512 + 128 cb + 32 w + {0, 16} + m; raw unit u of a super-block: row
+  // pass cb: columns it.col cols + 128 cb + 32 w + {0, 16} + m; raw unit u of a super-block: row
   // u / 9 (Q5_K: 11) of the wave's 32, the last load's upper lanes repeating the lower ones
-  const uint8_t* b0 = wd + (size_t)it.e * estride + (size_t)(it.col * kDownCols + 32 * wave) * rowb;
+  const uint8_t* b0 = wd + (size_t)it.e * estride + (size_t)(it.col * cols + 32 * wave) * rowb;
   constexpr int NL = raw_loads<FMT>(), kU = sb_bytes<FMT>() / 16;
   uint32_t uo[NL];
 #pragma unroll
@@ -457,8 +465,8 @@ __device__ __forceinline__ void down_item(const Item& it, const uint16_t* __rest
   constexpr int kB = Y16 ? 2 : 4;
   char* yb = reinterpret_cast<char*>(y) + (size_t)it.m0 * H * kB;
   const __amdgpu_buffer_rsrc_t rs = dma::rsrc(yb, it.rows * H * kB);
-  const int lane_off = (4 * g * H + it.col * kDownCols + 32 * wave + m) * kB;
-  for (int cb = 0; cb < kDownCols / kPassCols; ++cb) {
+  const int lane_off = (4 * g * H + it.col * cols + 32 * wave + m) * kB;
+  for (int cb = 0; cb < cols / kPassCols; ++cb) {
     f32x4_t acc[2][R];
 #pragma unroll
     for (int c = 0; c < 2; ++c)
@@ -471,7 +479,7 @@ __device__ __forceinline__ void down_item(const Item& it, const uint16_t* __rest
       // the next super-block: of these columns, or the first of the pass's next
       const bool row_end = sb + 1 == nsb;
       if (row_end) b0 += (size_t)kPassCols * rowb;
-      if (!row_end || cb + 1 < kDownCols / kPassCols) load_raw(b0 + (row_end ? 0 : (sb + 1) * sb_bytes<FMT>()));
+      if (!row_end || cb + 1 < cols / kPassCols) load_raw(b0 + (row_end ? 0 : (sb + 1) * sb_bytes<FMT>()));
       __builtin_amdgcn_sched_barrier(0);
       super_block<R, FMT>(wb, sm + sb * slot_bytes<R>(), m, g, acc);
     }
@@ -506,6 +514,7 @@ __global__ __launch_bounds__(512, (RMAX == 1 ? 4 : 2)) void k_gemm8_gateup(
     const int32_t* __restrict__ sorted_pairs, int K, int H, int I, int nsteps, uint16_t* __restrict__ S) {
   using namespace g8;
   Item it;
+  if (RMAX == 1 && few_tiles(tiles)) nsteps /= kGuFine;
   if (!get_item(tiles, offsets, I / (16 * nsteps), 16 * RMAX, it)) return;
   with_groups<RMAX>(it.rows, [&](auto R) {
     gateup_item<decltype(R)::value>(it, x16, wg, wu, estride, sorted_pairs, K, H, I, nsteps, S, g8_lds);
@@ -533,11 +542,12 @@ __global__ __launch_bounds__(64 * g8::kDnWaves, (RMAX == 1 ? 4 : 3)) void k_gemm
     return;
   }
   Item it;
-  if (!get_item(tiles, offsets, H / kDownCols, bm, it)) return;
+  const int cols = RMAX == 1 && few_tiles(tiles) ? kDownCols / kDnFine : kDownCols;
+  if (!get_item(tiles, offsets, H / cols, bm, it)) return;
   // a taller tile (the list is another kernel's) in pieces
   for (int left = it.rows; left > 0; left -= 16 * RMAX, it.m0 += 16 * RMAX) {
     it.rows = min(left, 16 * RMAX);
-    with_groups<RMAX>(it.rows, [&](auto R) { down_item<decltype(R)::value, FMT, Y16>(it, S, wd, estride, H, I, y, g8_lds); });
+    with_groups<RMAX>(it.rows, [&](auto R) { down_item<decltype(R)::value, FMT, Y16>(it, S, wd, estride, H, I, cols, y, g8_lds); });
     if (left > 16 * RMAX) __syncthreads();
   }
 }
@@ -546,9 +556,12 @@ __global__ __launch_bounds__(64 * g8::kDnWaves, (RMAX == 1 ? 4 : 3)) void k_gemm
 
 using namespace moe;
 
-// one block per (tile, slab): the tile list's capacity rounded up to whole groups of 8 tiles
-static dim3 g8_grid(int max_tiles, int ncol) {
-  return dim3((unsigned)((max_tiles + g8::kXcd - 1) / g8::kXcd * ncol * g8::kXcd));
+// one block per (tile, slab): the tile list's capacity rounded up to whole groups of 8 tiles; enough too for
+// a list of few tiles in `fine` times the slabs
+static dim3 g8_grid(int max_tiles, int ncol, int fine) {
+  static_assert(g8::kFewTiles % g8::kXcd == 0, "whole groups of 8 tiles");
+  const int n = (max_tiles + g8::kXcd - 1) / g8::kXcd * g8::kXcd;
+  return dim3((unsigned)(ncol * std::max(n, fine * std::min(n, g8::kFewTiles))));
 }
 
 bool moe_gemm8_gateup_supports(int fmt, int H, int I) {
@@ -568,7 +581,7 @@ int moe_launch_gemm8_gateup(const uint16_t* x16, const void* w_gate, const void*
   // tiles (one block on a CU, so the activations' load at its start is not covered by another):
   // 512 tokens 79 us, against 87 with 8
   const int ns = bm == 16 ? 8 : 16;
-  const dim3 grid = g8_grid(max_tiles, I / (16 * ns));
+  const dim3 grid = g8_grid(max_tiles, I / (16 * ns), bm == 16 ? g8::kGuFine : 1);
   const size_t lds = g8::kGuWaves * (size_t)(g8::wbuf_bytes<MOE_FMT_Q4_K>() + 2 * 2048 * (bm / 16));
   const uint8_t *g = reinterpret_cast<const uint8_t*>(w_gate), *u = reinterpret_cast<const uint8_t*>(w_up);
   if (bm == 16)
@@ -602,10 +615,10 @@ int moe_launch_gemm8_down(const uint16_t* S, const void* w_down, int fmt, size_t
     const int want = moe_shjob_down_blocks(job.T, job.H);
     if (job.n != want) return moe_set_error(MOE_E_ARG, "gemm8: %d shared-expert blocks given, %d needed", job.n, want);
   }
-  dim3 grid = g8_grid(max_tiles, H / g8::kDownCols);
+  const bool one = bm <= 16;
+  dim3 grid = g8_grid(max_tiles, H / g8::kDownCols, one ? g8::kDnFine : 1);
   grid.x += (unsigned)job.n;
   const uint8_t* w = reinterpret_cast<const uint8_t*>(w_down);
-  const bool one = bm <= 16;
   if (fmt == MOE_FMT_Q4_K)
     (one ? g8_down<1, MOE_FMT_Q4_K> : g8_down<2, MOE_FMT_Q4_K>)(y16, grid, st, S, w, expert_stride, tiles, offsets, bm, H, I, y, job);
   else

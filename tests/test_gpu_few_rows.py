@@ -63,6 +63,20 @@ def test_one_tile_height_or_the_other_same_bits(pkg, layer_q5k, dev):
     assert torch.isfinite(a).all() and torch.equal(a, b)
 
 
+@pytest.mark.parametrize("fixture", ["layer_c0", "layer_q5k"])
+def test_slab_count_does_not_change_the_bits(pkg, dev, request, fixture):
+    """16-row tile lists of 80 tiles (the finest slabs) and, with one token more, of 81 (whole ones)."""
+    lw, ow = request.getfixturevalue(fixture)
+    x = pkg.synth.make_input(17, seed=21, device=dev)
+    ids = torch.cat([torch.arange(80, dtype=torch.int32), torch.arange(48, dtype=torch.int32),
+                     torch.tensor([80] + list(range(48, 55)), dtype=torch.int32)]).view(17, 8)
+    a = _raw(pkg, lw, x[:16].contiguous(), ids[:16].contiguous().to(dev))
+    b = _raw(pkg, lw, x, ids.to(dev))
+    want = O.experts_and_combine(x[:16].cpu(), ids[:16].long(), torch.ones(16, 8, dtype=torch.bfloat16), ow)["expert_raw"]
+    assert torch.equal(a, b[:128])
+    assert _rel(a.view(16, 8, -1), want) <= 5e-4
+
+
 def test_large_and_small_activations(pkg, layer_c0, dev):
     """Rows whose sub-block sums pass 65504 (their SiLU rows saturate, here as on the other tiles), and
     small rows: x 0.05 gives SiLU rows of (0.05 0.9)^2 / 2 = 1e-3, still above f16's subnormals
